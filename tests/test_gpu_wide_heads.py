@@ -84,6 +84,55 @@ def test_wide_training_forward_outputs(batch, tokens_, heads, head_size):
     assert relative_rmse(to_np(bnd), bnd_ref) <= STATE_REL
 
 
+@pytest.mark.parametrize("head_size", [128, 256])
+@pytest.mark.parametrize("name,value", [("v", float("inf")), ("k", float("nan")),
+                                        ("a", float("-inf")), ("b", float("inf")),
+                                        ("decay_logits", float("nan")), ("r", float("nan"))])
+def test_wide_non_finite_token_leaves_the_tokens_before_it(head_size, name, value):
+    """A non-finite value in the middle of a 16-token chunk: what is finite token
+    by token (the earlier tokens of its chunk, the other columns where only v is
+    concerned, the other segments) is finite and right here too."""
+    C = require_gpu()
+    print(f"case wide non-finite D={head_size} {name}={value}", flush=True)
+    case = make_case(dtype=torch.bfloat16, head_size=head_size, lengths=(40, 48), num_heads=2,
+                     with_decay_bias=True, seed=head_size)
+    case[name][27, 1, 70] = value
+    C.handoff_fault_count(reset=True)
+    y_ref, pool_ref = oracle_expect(case)
+    out = wkv7(*tokens(case), state_pool=case["state_pool"], cu_seqlens=case["cu_seqlens"],
+               state_indices=case["state_indices"], decay_bias=case["decay_bias"])
+    torch.cuda.synchronize()
+    assert C.handoff_fault_count(reset=True) == 0
+    for got, want, rel in ((to_np(out), y_ref, 2.0e-3),
+                           (to_np(case["state_pool"]), pool_ref, STATE_REL)):
+        live = np.isfinite(want)
+        assert live.any() and np.array_equal(np.isfinite(got), live)
+        got, want = got[live].astype(np.float64), want[live]
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) <= rel
+
+
+def test_wide_training_forward_non_finite_token():
+    """sa and the state after every 16 tokens before and after a non-finite key."""
+    C = require_gpu()
+    case = make_case(dtype=torch.bfloat16, head_size=128, lengths=(48,), num_heads=1, seed=9)
+    case["k"][21, 0, 3] = float("inf")
+    x = [t.view(1, 48, 1, 128) for t in tokens(case)]
+    y = torch.empty_like(x[3])
+    bnd = torch.empty((1, 1, 3, 128, 128), device="cuda")
+    sa = torch.empty((1, 48, 1, 128), device="cuda")
+    C.pretrain_tmix_wkv7_recurrent_forward(*x, y, bnd, sa, 128)
+    torch.cuda.synchronize()
+    _, _, sa_ref, bnd_ref = oracle.wkv7_f64(*(to_np(t).reshape(48, 1, 128) for t in x),
+                                            cu_seqlens=np.array([0, 48], dtype=np.int32),
+                                            want_sa=True, boundary_len=16)
+    for got, want in ((to_np(sa).reshape(sa_ref.shape), sa_ref),
+                      (to_np(bnd).reshape(bnd_ref.shape), bnd_ref)):
+        live = np.isfinite(want)
+        assert live.any() and not live.all() and np.array_equal(np.isfinite(got), live)
+        assert relative_rmse(got[live], want[live]) <= STATE_REL
+    assert torch.isfinite(y[0, :21].float()).all()
+
+
 def test_wide_hand_off_give_up_fails_closed():
     """With the bounded waits' limit at zero polls the state waves give up at
     once: NaN outputs, the state untouched, one fault per workgroup, and the
