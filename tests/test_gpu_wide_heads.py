@@ -2,8 +2,9 @@
 against the fp64 oracle, around its 16-token chunks, its two sets of key waves
 (odd and even chunk counts), ragged and one-token segments, decay bias and
 scale, and with the training forward's outputs.  Final states meet 1e-6
-relative (fp32 sums of at most a few hundred terms, 2^-24 each); y meets the
-gates of the other kernels (its own 16-bit rounding dominates)."""
+relative (fp32 sums of at most a few hundred terms, 2^-24 each) and are no
+further from fp64 than a token-by-token fp32 evaluation; y meets the gates of
+the other kernels (its own 16-bit rounding dominates)."""
 
 from __future__ import annotations
 
@@ -82,6 +83,56 @@ def test_wide_training_forward_outputs(batch, tokens_, heads, head_size):
     assert_output_close(y.reshape(flat[0].shape), y_ref)
     assert relative_rmse(to_np(sa).reshape(sa_ref.shape), sa_ref) <= STATE_REL
     assert relative_rmse(to_np(bnd), bnd_ref) <= STATE_REL
+
+
+def _token_serial_f32(x):
+    """Final states and sa of [B, T, H, D] inputs from a zero state, token by token
+    in fp32 (sums over keys in pairs)."""
+    r, logits, k, v, a, b = (t.float() for t in x)
+    w = torch.exp(-float(np.exp(-0.5)) * torch.sigmoid(logits))
+    B, T, H, D = r.shape
+    state = torch.zeros((B, H, D, D), device=r.device)
+    sa = torch.empty((B, T, H, D), device=r.device)
+    for t in range(T):
+        parts = a[:, t, :, :, None] * state
+        while parts.shape[2] > 1:
+            parts = parts[:, :, 0::2] + parts[:, :, 1::2]
+        sa[:, t] = parts[:, :, 0]
+        state = w[:, t, :, :, None] * state + (
+            b[:, t, :, :, None] * sa[:, t, :, None, :] + k[:, t, :, :, None] * v[:, t, :, None, :])
+    return state, sa
+
+
+@pytest.mark.parametrize("decay", [(-6.0, -0.5), (-9.0, -4.0)])
+@pytest.mark.parametrize("head_size", [128, 256])
+def test_wide_training_forward_is_as_exact_as_token_by_token(head_size, decay):
+    """Errors against fp64 of the state after every 16 tokens and of sa, next to those
+    of a token-by-token fp32 evaluation of the same inputs.  Both are sums of
+    thousands of roundings, so their size is steady: a quarter more is allowed."""
+    C = require_gpu()
+    batch, tokens_, heads = 2, 256, 2
+    g = torch.Generator().manual_seed(head_size)
+    shape = (batch, tokens_, heads, head_size)
+    kk = torch.nn.functional.normalize(torch.randn(shape, generator=g), dim=-1)
+    p = torch.exp(torch.rand(shape, generator=g) * (decay[1] - decay[0]) + decay[0] + 0.5)
+    vals = [torch.randn(shape, generator=g), torch.logit(p.clamp(max=1 - 2.0 ** -23)),
+            torch.randn(shape, generator=g), torch.randn(shape, generator=g),
+            -kk, kk * torch.sigmoid(torch.randn(shape, generator=g))]
+    x = [t.to(torch.bfloat16).cuda() for t in vals]
+    y = torch.empty_like(x[3])
+    bnd = torch.empty((batch, heads, tokens_ // 16, head_size, head_size), device="cuda")
+    sa = torch.empty(shape, device="cuda")
+    C.pretrain_tmix_wkv7_recurrent_forward(*x, y, bnd, sa, head_size)
+    serial_state, serial_sa = _token_serial_f32(x)
+    flat = [to_np(t).reshape(batch * tokens_, heads, head_size) for t in x]
+    cu = np.arange(0, batch * tokens_ + 1, tokens_, dtype=np.int32)
+    _, _, sa_ref, bnd_ref = oracle.wkv7_f64(*flat, cu_seqlens=cu, want_sa=True, boundary_len=16)
+    for name, got, serial, want in (
+            ("state", bnd[:, :, -1], serial_state, bnd_ref.reshape(bnd.shape)[:, :, -1]),
+            ("sa", sa.reshape(sa_ref.shape), serial_sa.reshape(sa_ref.shape), sa_ref)):
+        err, limit = relative_rmse(to_np(got), want), 1.25 * relative_rmse(to_np(serial), want)
+        print(f"D={head_size} decay {decay} {name}: {err:.3e}, allowed {limit:.3e}", flush=True)
+        assert err <= limit
 
 
 @pytest.mark.parametrize("head_size", [128, 256])
