@@ -699,8 +699,12 @@ def dispatch_kernel_name(num_sequences: int, num_heads: int, head_size: int,
     io = "IoBF16" if dtype == torch.bfloat16 else "IoF16"
     name = _FAMILY_KERNELS[fam.value].format(io=io)
     if fam.value == N.KERNEL_SERIAL and head_size != 64:
-        wide = total_tokens >= 16 * num_sequences or max_seqlen >= 64
-        name = (f"chunk_wide_kernel<{head_size},{io}>" if wide
+        wide = ctypes.c_int32()
+        N.check(lib.fr2_wkv7_recurrent_fp32_wide_chunked(int(num_sequences), int(num_heads),
+                                                         int(head_size), int(total_tokens),
+                                                         int(max_seqlen), ctypes.byref(wide)),
+                "fr2_wkv7_recurrent_fp32_wide_chunked")
+        name = (f"chunk_wide_kernel<{head_size},{io}>" if wide.value
                 else f"serial_kernel<{head_size},{io},StF32>")
     return name
 

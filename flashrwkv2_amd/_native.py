@@ -62,6 +62,9 @@ SIGNATURES: dict[str, tuple] = {
     "fr2_wkv7_recurrent_fp32_dispatch": (
         c_int32, [c_int32, c_int32, c_int32, c_int64, c_int32, _i32p],
     ),
+    "fr2_wkv7_recurrent_fp32_wide_chunked": (
+        c_int32, [c_int32, c_int32, c_int32, c_int64, c_int32, _i32p],
+    ),
     "fr2_wkv7_prefill_split_plan": (
         c_int32, [c_int32] * 4 + [c_void_p] * 4),
     "fr2_wkv7_recurrent_fp32_split_plan": (

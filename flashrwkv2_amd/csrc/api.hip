@@ -33,7 +33,7 @@ using fr2::SegArgs;
 //     sequence exceeds twice the mean: a long sequence is one wave's serial
 //     chain there, and the workgroup-per-unit kernel finishes it sooner.
 // The token-serial kernel wins only within launch latency (U = 512, L = 5-8:
-// 0.0104 against 0.0114 ms).  D != 64 goes to launch_serial, which has its own
+// 0.0104 against 0.0114 ms).  D != 64 goes to launch_wide, which has its own
 // rule (token-serial or the fp32 chunked kernel).
 constexpr int kDecodeMaxSeqlen = 4;
 constexpr int kChunkMinSeqlen = 5;   // the smallest chunked threshold (U <= 256)
@@ -110,9 +110,11 @@ int run_family(int family, int D, int dtype, bool bf16_state, const SegArgs& p,
         if (rc != FR2_ERR_UNSUPPORTED) return rc;
       }
     }
+    if (family == kSerial && D != 64 && !bf16_state)
+      return fr2::launch_wide(D, dtype, p, nseg, s, max_seqlen);
   }
   switch (family) {
-    case kSerial: return fr2::launch_serial(D, dtype, bf16_state, p, nseg, s, max_seqlen);
+    case kSerial: return fr2::launch_serial(D, dtype, bf16_state, p, nseg, s);
     case kDecode:
       if (bf16_state) return FR2_ERR_UNSUPPORTED;
       return fr2::launch_decode(D, dtype, p, nseg, s);
@@ -180,6 +182,17 @@ extern "C" int fr2_wkv7_recurrent_fp32_dispatch(int32_t num_sequences, int32_t n
   if (f == kChunkedWave && fr2::wave_longest_first(num_sequences, max_seqlen, total_tokens))
     f = 5;
   *kernel = f;
+  return FR2_OK;
+}
+
+extern "C" int fr2_wkv7_recurrent_fp32_wide_chunked(int32_t num_sequences, int32_t num_heads,
+                                                    int32_t head_size, int64_t total_tokens,
+                                                    int32_t max_seqlen, int32_t* chunked) {
+  if (chunked == nullptr || num_sequences <= 0 || num_sequences > 65535 || num_heads <= 0 ||
+      total_tokens <= 0)
+    return FR2_ERR_INVALID_ARGUMENT;
+  if (head_size != 64 && head_size != 128 && head_size != 256) return FR2_ERR_UNSUPPORTED;
+  *chunked = fr2::wide_chunked(head_size, num_sequences, num_heads, total_tokens, max_seqlen);
   return FR2_OK;
 }
 
@@ -499,15 +512,16 @@ extern "C" int fr2_wkv7_pretrain_forward_split(int32_t batch, int32_t tokens,
   p.boundary_len = 16;
   p.boundary_per_seg = tokens / 16;
   // D = 64 runs the chunked MFMA kernel, which emits sa and the post-chunk
-  // states of its 16-token chunks directly; other head sizes run token-serial
+  // states of its 16-token chunks directly; the other head sizes have their own
+  // kernels
   if (head_size == 64) {
     fr2::set_train_split(p, batch, tokens, split_workspace);
     const int rc = fr2::launch_chunked(FR2_DTYPE_BFLOAT16, p, batch, tokens,
                                        static_cast<hipStream_t>(stream));
     if (rc != FR2_ERR_UNSUPPORTED) return rc;
   }
-  return fr2::launch_serial(head_size, FR2_DTYPE_BFLOAT16, false, p, batch,
-                            static_cast<hipStream_t>(stream));
+  return fr2::launch_wide(head_size, FR2_DTYPE_BFLOAT16, p, batch,
+                          static_cast<hipStream_t>(stream));
 }
 
 extern "C" int fr2_wkv7_pretrain_forward(int32_t batch, int32_t tokens,
@@ -714,8 +728,7 @@ extern "C" int fr2_wkv7_rl_infctx_replay(
   // serial; 65 536 units, L = 16: 0.62 vs 0.90 ms decode)
   if (head_size == 64)
     return fr2::launch_chunked_wave(dtype, p, num_chunks, 0, static_cast<hipStream_t>(stream));
-  return fr2::launch_serial(head_size, dtype, false, p, num_chunks,
-                            static_cast<hipStream_t>(stream));
+  return fr2::launch_wide(head_size, dtype, p, num_chunks, static_cast<hipStream_t>(stream));
 }
 
 // ---------------------------------------------------------------------------

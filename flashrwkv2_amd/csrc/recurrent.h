@@ -137,9 +137,13 @@ __host__ __device__ inline void split_piece(const SegArgs& p, int n, int j, int&
   len = j == 0 ? lead : p.split_len;
 }
 
-// max_seqlen: the longest segment, where known (a hint of the choice of kernel)
 int launch_serial(int D, int dtype, bool bf16_state, const SegArgs& p, int nseg,
-                  hipStream_t s, int max_seqlen = 0);
+                  hipStream_t s);
+// Head sizes 128 and 256, fp32 state: chunked (launch_chunked_wide) where
+// wide_chunked says so, else token-serial.  max_seqlen: the longest segment, where
+// known (0: unknown).
+bool wide_chunked(int D, int64_t nseg, int64_t H, int64_t tokens, int max_seqlen);
+int launch_wide(int D, int dtype, const SegArgs& p, int nseg, hipStream_t s, int max_seqlen = 0);
 int launch_decode(int D, int dtype, const SegArgs& p, int nseg, hipStream_t s);
 // FP16 state pool with the Albatross delta update (fp16 tokens), followed by
 // the elapsed-count advance of every active sequence's slot.

@@ -11,7 +11,9 @@
 //  csrc/sm120/tmix/wkv7/infer_recurrent_fp32io16_forward_varlen.cu:90-192).
 #include "recurrent.h"
 
+#include <algorithm>
 #include <array>
+#include <cmath>
 #include <type_traits>
 
 namespace fr2 {
@@ -957,28 +959,55 @@ int launch_advance_elapsed(const SegArgs& p, int nseg, int32_t* elapsed, hipStre
   return record_launch();
 }
 
-// Head sizes 128 and 256, fp32 state: the chunked kernel (chunk_wide.hip) from a
-// mean of 16 tokens per segment on, or when one segment is long enough for its
-// serial chain to outlast the rest; the token-serial kernel for shorter ones.
-// us, token-serial against chunked, D = 128: 512 units of 8 tokens 23.9 / 34.7,
-// of 16 tokens 38.3 / 36.0, of 24 tokens 51.9 / 48.1; 2 048 units of 12 tokens
-// 103 / 119, of 16 tokens 128 / 119; 128 units of 16 tokens 21.7 / 12.3.
+// Head sizes 128 and 256, fp32 state: the chunked kernel (chunk_wide.hip) where a
+// mean of 16 tokens per segment or a segment of 64 makes it worth a look and the
+// measured costs (us) say that it is the faster one:
+//   token-serial, u = units / 256: a unit alone takes 1.05 us a token at D = 128
+//     (3.15 at D = 256); with more than one per CU they cost u times
+//     max(5.2, 2.7 + 0.79 tokens) (24 + 3.2 tokens); a segment longer than the
+//     mean adds its chain;
+//   chunked: each workgroup (D / 64 per unit, one per CU) 4.6 and 3.4 (6.9) per
+//     chunk, a whole one for a partial one; the longest adds its chunks.
+// The two cross where chunks are mostly padding.  us, token-serial against chunked,
+// D = 128: 512 units of 16 tokens 37 / 35, of 17 tokens 40 / 47, of 24 50 / 47; 4 096
+// units of 16 tokens 248 / 253, of 17 275 / 354, of 32 434 / 360; one segment of 64
+// tokens (256) among 4 095 units of one 155 / 252 (370 / 292), among 511 77 / 43.
+// D = 256 differs only where 4 096 units have one token each: 652 / 751.
 constexpr int kWideChunkTokens = 16;
 constexpr int kWideChunkLongest = 64;
 
+bool wide_chunked(int D, int64_t nseg, int64_t H, int64_t tokens, int max_seqlen) {
+  // max_seqlen may be a capacity: where every segment has a token, the longest has
+  // what the others leave.  (Unknown, it counts as the mean.)
+  const int64_t most = std::min<int64_t>(max_seqlen, tokens - nseg + 1);
+  if (D == 64 || (tokens < kWideChunkTokens * nseg && most < kWideChunkLongest)) return false;
+  const double mean = static_cast<double>(tokens) / nseg;
+  const double longest = std::max(mean, static_cast<double>(most));
+  const double u = nseg * H / 256.0, groups = std::max(1.0, u * (D / 64));
+  const double token_us = D == 128 ? 1.05 : 3.15, chunk_us = D == 128 ? 3.4 : 6.9;
+  const double shared = D == 128 ? std::max(5.2, 2.7 + 0.79 * mean) : 24.0 + 3.2 * mean;
+  const double serial = (D == 128 ? 5.0 : 8.0) + std::max(u * shared, token_us * mean) +
+                        token_us * (longest - mean);
+  const double chunks = longest > mean ? std::max(1.0, mean / 16 + 0.5) : std::ceil(mean / 16);
+  const double chunked = 1.5 + groups * (4.6 + chunk_us * chunks) +
+                         chunk_us * std::max(0.0, std::ceil(longest / 16) - chunks);
+  return chunked < serial;
+}
+
+int launch_wide(int D, int dtype, const SegArgs& p, int nseg, hipStream_t s, int max_seqlen) {
+  const int64_t tokens = p.out_elems / (static_cast<int64_t>(p.num_heads) * D);
+  if (wide_chunked(D, nseg, p.num_heads, tokens, max_seqlen)) {
+    const int rc = launch_chunked_wide(D, dtype, p, nseg, s);
+    if (rc != FR2_ERR_UNSUPPORTED) return rc;
+  }
+  return launch_serial(D, dtype, false, p, nseg, s);
+}
+
 int launch_serial(int D, int dtype, bool bf16_state, const SegArgs& p, int nseg,
-                  hipStream_t s, int max_seqlen) {
+                  hipStream_t s) {
   if (bf16_state) {
     if (dtype != FR2_DTYPE_BFLOAT16) return FR2_ERR_UNSUPPORTED;
     return launch_serial_io<IoBF16, StBF16>(D, p, nseg, s);
-  }
-  if (D != 64) {
-    const int64_t tokens = p.out_elems / (static_cast<int64_t>(p.num_heads) * D);
-    if (tokens >= kWideChunkTokens * static_cast<int64_t>(nseg) ||
-        max_seqlen >= kWideChunkLongest) {
-      const int rc = launch_chunked_wide(D, dtype, p, nseg, s);
-      if (rc != FR2_ERR_UNSUPPORTED) return rc;
-    }
   }
   if (dtype == FR2_DTYPE_BFLOAT16) return launch_serial_io<IoBF16, StF32>(D, p, nseg, s);
   if (dtype == FR2_DTYPE_FLOAT16) return launch_serial_io<IoF16, StF32>(D, p, nseg, s);

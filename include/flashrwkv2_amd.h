@@ -181,6 +181,16 @@ int fr2_wkv7_recurrent_fp32_dispatch(int32_t num_sequences, int32_t num_heads,
                                      int32_t max_seqlen, int32_t* kernel);
 
 /*
+ * Whether fr2_wkv7_recurrent_fp32_forward runs a launch of this shape at
+ * head_size 128 or 256 on the fp32 chunked kernel (*chunked = 1) or token-serial
+ * (0; always at head_size 64): the choice behind dispatch's 0.  Pure host
+ * computation, as above; no reference counterpart.
+ */
+int fr2_wkv7_recurrent_fp32_wide_chunked(int32_t num_sequences, int32_t num_heads,
+                                         int32_t head_size, int64_t total_tokens,
+                                         int32_t max_seqlen, int32_t* chunked);
+
+/*
  * Sequence-split plan for the chunked prefill (head_size 64).  With few
  * (sequence, head) units one block per unit leaves most of the GPU idle; the
  * plan cuts every sequence into up to *pieces pieces: piece 0 of *lead_len

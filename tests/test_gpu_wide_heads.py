@@ -27,6 +27,7 @@ pytestmark = pytest.mark.gpu
 
 from flashrwkv2_amd.tmix.wkv7 import (  # noqa: E402
     infer_tmix_wkv7_recurrent_fp32io16_forward_varlen as wkv7,
+    prepare_tmix_wkv7_recurrent_metadata as prepare,
 )
 
 STATE_REL = 1.0e-6
@@ -184,27 +185,60 @@ def test_wide_training_forward_non_finite_token():
     assert torch.isfinite(y[0, :21].float()).all()
 
 
-def test_wide_hand_off_give_up_fails_closed():
+@pytest.mark.parametrize("head_size", [128, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_hand_off_give_up_fails_closed(head_size, dtype):
     """With the bounded waits' limit at zero polls the state waves give up at
     once: NaN outputs, the state untouched, one fault per workgroup, and the
-    same call is right again with the limit restored."""
+    same call is right again with the limit restored.  The token-serial kernel,
+    forced, has no hand-off: no fault."""
     C = require_gpu()
-    case = make_case(dtype=torch.bfloat16, head_size=128, lengths=(64, 40), num_heads=2, seed=3)
+    case = make_case(dtype=dtype, head_size=head_size, lengths=(64, 40), num_heads=2, seed=3)
     pool = case["state_pool"]
     before = pool.clone()
+    ticket = prepare(case["cu_seqlens"], case["state_indices"], total_tokens=104,
+                     state_pool_size=pool.shape[0])
+    serial_pool, serial = pool.clone(), torch.empty_like(case["v"])
     C.handoff_fault_count(reset=True)
     C._set_handoff_spin_limit(0)
     try:
+        C.tmix_wkv7_recurrent_fp32_kernel_forced(0, case["cu_seqlens"], case["state_indices"],
+                                                 serial_pool, *tokens(case), serial, 1.0, None,
+                                                 ticket)
+        torch.cuda.synchronize()
+        assert C.handoff_fault_count(reset=True) == 0
         out = wkv7(*tokens(case), state_pool=pool, cu_seqlens=case["cu_seqlens"],
                    state_indices=case["state_indices"])
         torch.cuda.synchronize()
     finally:
         C._set_handoff_spin_limit(-1)
     assert torch.isnan(out.float()).all() and torch.equal(pool, before)
-    assert C.handoff_fault_count(reset=True) == 2 * 2 * 2   # sequences x heads x column halves
+    # sequences x heads x groups of 64 columns
+    assert C.handoff_fault_count(reset=True) == 2 * 2 * (head_size // 64)
     y_ref, _ = oracle_expect(case)
+    assert_output_close(serial, y_ref)
     out = wkv7(*tokens(case), state_pool=pool, cu_seqlens=case["cu_seqlens"],
                state_indices=case["state_indices"])
     torch.cuda.synchronize()
     assert_output_close(out, y_ref)
     assert C.handoff_fault_count(reset=True) == 0
+
+
+@pytest.mark.parametrize("head_size", [128, 256])
+def test_wide_training_forward_give_up_fails_closed(head_size):
+    """The form with sa and the 16-token states: NaN in y and sa, counted."""
+    C = require_gpu()
+    x = [t.view(1, 64, 2, head_size) for t in tokens(make_case(head_size=head_size, lengths=(64,),
+                                                               num_heads=2, seed=4))]
+    y = torch.zeros_like(x[3])
+    bnd = torch.empty((1, 2, 4, head_size, head_size), device="cuda")
+    sa = torch.zeros((1, 64, 2, head_size), device="cuda")
+    C.handoff_fault_count(reset=True)
+    C._set_handoff_spin_limit(0)
+    try:
+        C.pretrain_tmix_wkv7_recurrent_forward(*x, y, bnd, sa, head_size)
+        torch.cuda.synchronize()
+    finally:
+        C._set_handoff_spin_limit(-1)
+    assert C.handoff_fault_count(reset=True) == 2 * (head_size // 64)
+    assert torch.isnan(y.float()).all() and torch.isnan(sa).all()

@@ -198,6 +198,37 @@ def test_dispatch_query_reports_the_policy(lib, n, h, d, total, maxlen, want):
     assert fam.value == want
 
 
+@pytest.mark.parametrize("n,h,d,total,maxlen,chunked", [
+    (8, 16, 128, 8 * 2048, 2048, True),
+    (32, 16, 128, 32 * 16, 16, True),           # 512 units of one whole chunk
+    (32, 16, 128, 32 * 17, 17, False),          # ... and of one token more: half padding
+    (64, 16, 128, 64 * 20, 20, False),
+    (32, 16, 128, 31 + 64, 64, True),           # one longer sequence among few
+    (256, 16, 128, 255 + 64, 64, False),        # ... among many short ones
+    (256, 16, 128, 255 + 1024, 1024, True),
+    (256, 16, 128, 256, 4096, False),           # decode on a ticket with a large capacity
+    (128, 8, 256, 128 * 17, 17, True),
+    (512, 8, 256, 511 + 64, 64, False),
+    (8, 32, 128, 8 * 15, 15, False),
+    (8, 32, 128, 8 * 4096, 0, True),            # unknown longest sequence: the mean
+    (8, 32, 64, 8 * 4096, 4096, False),
+])
+def test_wide_head_rule_follows_the_measured_costs(lib, n, h, d, total, maxlen, chunked):
+    import ctypes
+
+    from flashrwkv2_amd import _C
+
+    assert _C.dispatch_kernel_name(n, h, d, total, maxlen).startswith("chunk_wide") == chunked
+    got = ctypes.c_int32(-1)
+    assert lib.fr2_wkv7_recurrent_fp32_wide_chunked(n, h, d, total, maxlen,
+                                                    ctypes.byref(got)) == 0
+    assert got.value == int(chunked)
+    assert lib.fr2_wkv7_recurrent_fp32_wide_chunked(0, h, d, total, maxlen, ctypes.byref(got)) == \
+        N.FR2_ERR_INVALID_ARGUMENT
+    assert lib.fr2_wkv7_recurrent_fp32_wide_chunked(n, h, 96, total, maxlen,
+                                                    ctypes.byref(got)) == N.FR2_ERR_UNSUPPORTED
+
+
 def test_dispatch_query_rejects_bad_arguments(lib):
     import ctypes
     fam = ctypes.c_int32(-1)
