@@ -957,6 +957,10 @@ extern "C" int fr2_wkv7_statetune_padded_backward(
                                                static_cast<hipStream_t>(stream));
 }
 
+namespace {
+constexpr int32_t kMaxRowSequences = 65535;
+}  // namespace
+
 // Lays a StateTune chunk list (host arrays) out as row blocks for
 // fr2_wkv7_statetune_rows_forward / _backward (D = 64, bf16): every chunk cut
 // into 16-row blocks from its first row, its last block shorter where 16 does not
@@ -965,9 +969,9 @@ extern "C" int fr2_wkv7_statetune_padded_backward(
 //   chunk_seq [C], chunk_block [C], seq_first_chunk [B]
 // and info = {blocks, spans, blocks per span, most blocks of a sequence}.
 // Returns the table's length; 0 when the list does not suit it (offsets that do
-// not cover the list, rows out of range or in two chunks, no tokens, or more than
-// four times the tokens in blocks: many tiny chunks run faster token-serial); -1 for an
-// invalid argument, -2 when `capacity` (ints) is too small.
+// not cover the list, rows out of range or in two chunks, no tokens, more than
+// four times the tokens in blocks: many tiny chunks run faster token-serial, or more
+// sequences, chunks or spans than a grid holds); -1 for an invalid argument, -2 when `capacity` (ints) is too small.
 // 4 * (T / 16 + C) + 3 * (B + 1) + 2 * C ints always suffice.
 extern "C" int64_t fr2_wkv7_statetune_rows_plan(
     const int32_t* sequence_chunk_offsets, const int32_t* chunk_token_starts,
@@ -978,6 +982,9 @@ extern "C" int64_t fr2_wkv7_statetune_rows_plan(
   if (!off || !st || !en || !table || !info ||
       !statetune_sizes_ok(num_sequences, num_chunks, total_tokens, num_heads))
     return -1;
+  // what the launches' grids cannot hold stays token-serial too: sequences are the
+  // ring kernel's grid.y, (chunk, head) and (span, head) pairs one-dimensional grids
+  if (B > kMaxRowSequences || static_cast<int64_t>(C) * num_heads > 0x7fffffff) return 0;
   if (off[0] != 0 || off[B] != C) return 0;
   for (int b = 0; b < B; ++b)
     if (off[b + 1] < off[b] || off[b + 1] > C) return 0;
@@ -1019,6 +1026,7 @@ extern "C" int64_t fr2_wkv7_statetune_rows_plan(
   const int every = fr2::key_block_span(seq_blocks, B, num_heads);
   int64_t num_spans = 0;
   for (int b = 0; b < B; ++b) num_spans += (seq_blocks[b + 1] - seq_blocks[b] + every - 1) / every;
+  if (num_spans * num_heads > 0x7fffffff) return 0;
   const int64_t total = 2 * blocks + 2 * (B + 1) + 2 * num_spans + 2 * static_cast<int64_t>(C) + B;
   if (capacity < total) return -2;
   int32_t* const seq_spans = seq_blocks + B + 1;
@@ -1065,7 +1073,7 @@ bool statetune_rows_ok(int32_t num_sequences, int32_t num_chunks, int64_t total_
                        int32_t num_heads, const int32_t* table, const int32_t* info) {
   // info's fields in the ranges fr2_wkv7_statetune_rows_plan writes
   return statetune_sizes_ok(num_sequences, num_chunks, total_tokens, num_heads) &&
-         num_sequences <= 65535 && table && info && info[0] >= 1 &&
+         num_sequences <= kMaxRowSequences && table && info && info[0] >= 1 &&
          info[0] <= total_tokens / 16 + num_chunks && info[1] >= 1 && info[1] <= info[0] &&
          info[2] >= 1 && info[3] >= 1 && info[3] <= info[0];
 }

@@ -65,6 +65,16 @@ def test_rows_match_the_padded_grid(seed):
         (b, i) for b in range(B) for i in range(seq_spans[b + 1] - seq_spans[b])]
 
 
+@pytest.mark.parametrize("B,H", [(65535, 1), (65536, 1), (40000, 60000)])
+def test_more_sequences_or_chunks_than_a_grid_holds(B, H):
+    """Such a list is left to the token-serial kernels, which take it."""
+    ends = np.arange(1, B + 1, dtype=np.int32) * 16
+    ends[-1] += 1   # (not uniform)
+    meta = np.concatenate([np.arange(B + 1), ends[:1] * 0, ends[:-1], ends]).astype(np.int32)
+    rows = statetune_rows_plan(meta, B, B, int(ends[-1]), H)
+    assert (rows is not None) == (B == 65535)
+
+
 @pytest.mark.parametrize("offsets,starts,ends,T", [
     ([0, 1, 2], [0, 48], [64, 112], 112),          # rows in two chunks
     ([0, 1, 2], [0, 64], [64, 129], 128),          # past the end
