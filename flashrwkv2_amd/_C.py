@@ -112,11 +112,12 @@ def _set_handoff_spin_limit(polls: int) -> None:
             "fr2_debug_set_handoff_spin_limit")
 
 
-def _set_handoff_stall(on: bool) -> None:
+def _set_handoff_stall(on: int) -> None:
     """Test hook: while on, the chunked kernel's key waves never publish their
     operators, so every block stalls at its first operator wait and fails
-    closed after the spin limit."""
-    N.check(N.load().fr2_debug_set_handoff_stall(int(bool(on))), "fr2_debug_set_handoff_stall")
+    closed after the spin limit (2: only a sequence split's later pieces but the
+    last, 3: only its summaries)."""
+    N.check(N.load().fr2_debug_set_handoff_stall(int(on)), "fr2_debug_set_handoff_stall")
 
 
 def _set_chunk_ring(on: bool) -> None:

@@ -375,7 +375,7 @@ extern "C" int fr2_wkv7_recurrent_fp32_forward_split_noalloc(
   if (need > kNoAllocScratchFloats) {
     fr2::set_last_error(
         "fr2_wkv7_recurrent_fp32_forward_split_noalloc: the split's workspace exceeds the "
-        "16 MiB no-allocation scratch (num_sequences * (3 pieces - 2) * num_heads * 16 KiB)");
+        "16 MiB no-allocation scratch (num_sequences * num_heads * ((2 pieces - 2) * 16 KiB + 4 pieces))");
     return FR2_ERR_INVALID_ARGUMENT;
   }
   float* ws = scratch_address();
@@ -1357,10 +1357,10 @@ extern "C" int fr2_debug_set_chunk_ring(int32_t on) {
 }
 
 // Test hook: while on, the chunked kernel's key waves never publish their
-// operators to the state waves, so every block stalls at its first
-// operator wait and, after the spin limit, fails closed; every kernel still
-// runs to its end.
+// operators to the state waves, so every block (2: a sequence split's later
+// pieces but the last; 3: its summaries) stalls at its first operator wait and,
+// after the spin limit, fails closed; every kernel still runs to its end.
 extern "C" int fr2_debug_set_handoff_stall(int32_t on) {
-  fr2::set_handoff_stall(on != 0);
+  fr2::set_handoff_stall(on == 2 || on == 3 ? on : on != 0);
   return FR2_OK;
 }

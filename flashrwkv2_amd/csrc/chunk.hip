@@ -919,7 +919,7 @@ __global__ __launch_bounds__(NT) void chunk64_kernel(SegArgs p) {
       signal(&sm.part1[kw], gn + 1);
       wait_ge(&sm.part1[partner], gn + 1, p.spin_limit, &sm.fault);
       if (active) key_part2<kVExact>(sm, sm.ops[par][cc], par, cc, hh, i, q, kr);
-      if (!p.handoff_stall) signal(&sm.ready[kw], gn + 1);
+      if (p.handoff_stall != 1) signal(&sm.ready[kw], gn + 1);
     };
     for (int gn = 0; gn < ngroups; gn += 2) {
       iter(std::integral_constant<int, 0>{}, rawA, rawB, gn);
@@ -963,6 +963,7 @@ struct alignas(16) SmemR {
   // finished
   int ready[kKeyW], consumed[4];
   int fault;
+  int lost;                           // the start state came from a block that failed
 };
 
 // A chunk's outputs on their way to memory: the post-chunk state, sa and y, each
@@ -1279,6 +1280,62 @@ __device__ __forceinline__ float* split_summary_of(const SegArgs& p, int seg, in
 __device__ __forceinline__ f32x4* split_tile(float* blk, int a, int b, int lane) {
   return reinterpret_cast<f32x4*>(blk) + (4 * a + b) * 64 + lane;
 }
+// The failure words of a split segment: word 0 for its first piece and word m for
+// the summary of piece m, written by those blocks (0 or 1), and the last word, which
+// the first piece clears for the second launch's blocks.  There, a block whose start
+// state is chained from a failed one fails too; and a state updated in place stays
+// untouched when another piece of its segment fails, before or after the last piece
+// stored it: whichever of the two comes second to the word puts the saved state back.
+constexpr int kStateStored = 1, kPieceFailed = 2;
+__device__ __forceinline__ int* split_flags_of(const SegArgs& p, int seg, int h) {
+  return p.split_flags + (static_cast<int64_t>(seg) * p.num_heads + h) * p.split_pieces;
+}
+__device__ __forceinline__ float* split_saved_of(const SegArgs& p, int seg, int h) {
+  return p.split_saved + (static_cast<int64_t>(seg) * p.num_heads + h) * D * D;
+}
+// State columns [16 w, 16 w + 16) of the slot at sbase; kThrough: past the XCD's L2,
+// so that a block on another XCD may overwrite them.
+template <bool kThrough>
+__device__ __forceinline__ void store_state(const SegArgs& p, int64_t sbase, int w, int lane,
+                                            const f32x4 (&S)[4]) {
+  const int64_t at = sbase + (4 * (lane >> 4)) * D + 16 * w + (lane & 15);
+  auto put = [](auto* to, auto x) {
+    if constexpr (kThrough)
+      __hip_atomic_store(to, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+      *to = x;
+  };
+  if (p.state_bf16) {
+    uint16_t* const to = static_cast<uint16_t*>(p.state_out) + at;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) put(to + (16 * kb + e) * D, IoBF16::from_f32(S[kb][e]));
+  } else {
+    float* const to = static_cast<float*>(p.state_out) + at;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) put(to + (16 * kb + e) * D, S[kb][e]);
+  }
+}
+// (one wave) Adds `mine` to the segment's last word; where `other` came first, the
+// saved state goes back to the slot.
+__device__ __forceinline__ void settle_state(const SegArgs& p, int seg, int h, int64_t sbase,
+                                             int lane, int mine, int other) {
+  int seen = 0;
+  if (lane == 0)
+    seen = __hip_atomic_fetch_or(split_flags_of(p, seg, h) + p.split_pieces - 1, mine,
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((__builtin_amdgcn_readfirstlane(seen) & other) == 0) return;
+  float* const saved = split_saved_of(p, seg, h);
+  for (int w = 0; w < 4; ++w) {
+    f32x4 S[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) S[kb] = *split_tile(saved, w, kb, lane);
+    store_state<true>(p, sbase, w, lane, S);
+  }
+}
 
 // Start state of piece j >= 1 for this wave's 16 columns: the state after
 // piece 0, carried over pieces 1..j-1 by S <- Phi_m S + F_m on the fp32 matrix
@@ -1393,9 +1450,12 @@ __device__ __forceinline__ void ring_real(const SegArgs& p,
     return bnd_base != nullptr && snap_at(c) % p.boundary_every == 0;
   };
 
-  if (tid < kKeyW + 5) (&sm.ready[0])[tid] = 0;
+  if (tid < kKeyW + 6) (&sm.ready[0])[tid] = 0;
   __syncthreads();   // the only workgroup barrier before the end: counters are zero
 
+  // (split) the state is updated in place, by the last piece
+  const bool in_place =
+      kPhase != kWhole && p.state_in != nullptr && p.state_out == p.state_in;
   const int vcol = 16 * (wv & 3) + i;
   const int64_t sbase = (static_cast<int64_t>(slot) * H + h) * D * D;
   if (wv < 4) {
@@ -1404,7 +1464,15 @@ __device__ __forceinline__ void ring_real(const SegArgs& p,
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) S[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (kPhase == kRest) {
+      // (requested in front of the chain's blocks, used when those have arrived)
+      const int* const flags = split_flags_of(p, seg, h);
+      int lost = flags[min(lane, piece - 1)];
       chain_start_state(p, seg, piece, h, wv, lane, S);
+      for (int m = lane + 64; m < piece; m += 64) lost |= flags[m];
+      if (lost != 0) {
+        raise_fault(&sm.lost);
+        raise_fault(&sm.fault);
+      }
     } else if (p.state_in != nullptr && p.state_bf16) {
       // (bf16-state contract) widened once; the state stays fp32 for the
       // whole call and is rounded back once at the end
@@ -1419,6 +1487,11 @@ __device__ __forceinline__ void ring_real(const SegArgs& p,
       for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[kb][e] = sin[(kb * 16 + 4 * q + e) * D];
+    }
+    if (kPhase == kLead && in_place && !pc.last) {
+      float* const saved = split_saved_of(p, seg, h);
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) *split_tile(saved, wv, kb, lane) = S[kb];
     }
     // Each state wave writes its own 16 output columns: the chunk's rows are
     // staged in the wave's column band of yb (2-byte stores from the
@@ -1461,10 +1534,23 @@ __device__ __forceinline__ void ring_real(const SegArgs& p,
       signal(&sm.consumed[wv], c + 1);
     }
     __syncthreads();
-    if (peek(&sm.fault) != 0) {
-      if (tid == 0 && p.handoff_fault != nullptr) atomicAdd(p.handoff_fault, 1);
+    const bool failed = peek(&sm.fault) != 0;
+    if (kPhase == kLead && !pc.last && tid == 0) {
+      int* const flags = split_flags_of(p, seg, h);
+      flags[0] = failed;
+      flags[p.split_pieces - 1] = 0;
+    }
+    if (failed) {
+      const bool lost = kPhase == kRest && peek(&sm.lost) != 0;
+      if (tid == 0 && !lost && p.handoff_fault != nullptr) atomicAdd(p.handoff_fault, 1);
       const float qnan = quiet_nan();
       const raw nanv = Io::from_f32(qnan);
+      if (kRev && pc.last && p.state_out != nullptr) {   // (an output of its own there)
+        float* const sout = static_cast<float*>(p.state_out) + sbase;
+        for (int e = tid; e < D * D; e += 256) sout[e] = qnan;
+      }
+      if (kPhase == kRest && in_place && !pc.last && !lost && wv == 0)
+        settle_state(p, seg, h, sbase, lane, kPieceFailed, kStateStored);
       for (int64_t e = tid; e < static_cast<int64_t>(t1 - t0) * D; e += 256) {
         const int pos = static_cast<int>(e / D), col = static_cast<int>(e % D);
         BlockRow yr{t0 + pos, true}, ur{0, true};
@@ -1493,19 +1579,15 @@ __device__ __forceinline__ void ring_real(const SegArgs& p,
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) *split_tile(sout, wv, kb, lane) = S[kb];
       }
-    } else if (p.state_out != nullptr && p.state_bf16) {
-      uint16_t* soutb = static_cast<uint16_t*>(p.state_out) + sbase + vcol;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          soutb[(kb * 16 + 4 * q + e) * D] = IoBF16::from_f32(S[kb][e]);
+    } else if (kPhase == kRest && in_place) {
+      store_state<true>(p, sbase, wv, lane, S);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the stores have landed
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __syncthreads();                      // (with the key waves)
+      if (wv == 0) settle_state(p, seg, h, sbase, lane, kStateStored, kPieceFailed);
     } else if (p.state_out != nullptr) {
-      float* sout = static_cast<float*>(p.state_out) + sbase + vcol;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sout[(kb * 16 + 4 * q + e) * D] = S[kb][e];
+      store_state<false>(p, sbase, wv, lane, S);
     }
   } else {
     // ---------------- key waves: whole chunks kw, kw + 4, ...
@@ -1685,9 +1767,11 @@ __device__ __forceinline__ void ring_real(const SegArgs& p,
       }
       if (c + kKeyW < nchunks) load_chunk(c + kKeyW);
       key_blocks_ring(op, acc, i, q);
-      if (!p.handoff_stall) signal(&sm.ready[kw], (c - kw) / kKeyW + 1);
+      if (p.handoff_stall != 1 && !(p.handoff_stall == 2 && kPhase == kRest && !pc.last))
+        signal(&sm.ready[kw], (c - kw) / kKeyW + 1);
     }
     __syncthreads();   // pairs with the state waves' final barrier
+    if (kPhase == kRest && in_place && pc.last && peek(&sm.fault) == 0) __syncthreads();
   }
 }
 
@@ -1747,7 +1831,9 @@ __device__ __forceinline__ void ring_summary(const SegArgs& p,
     __syncthreads();
     float* sout = split_summary_of(p, seg, piece, 0, h);
     float* pout = split_summary_of(p, seg, piece, 1, h);
-    if (peek(&sm.fault) != 0) {
+    const bool failed = peek(&sm.fault) != 0;
+    if (tid == 0) split_flags_of(p, seg, h)[piece] = failed;
+    if (failed) {
       // the pieces that start from this summary come out NaN as well
       if (tid == 0 && p.handoff_fault != nullptr) atomicAdd(p.handoff_fault, 1);
       const float qnan = quiet_nan();
@@ -1840,7 +1926,7 @@ __device__ __forceinline__ void ring_summary(const SegArgs& p,
       }
       if (c + kKeyW < nchunks) load_chunk(c + kKeyW);
       key_blocks_ring_sum(op, acc, i, q);
-      if (!p.handoff_stall) signal(&sm.ready[kw], (c - kw) / kKeyW + 1);
+      if (p.handoff_stall != 1 && p.handoff_stall != 3) signal(&sm.ready[kw], (c - kw) / kKeyW + 1);
     }
     __syncthreads();   // pairs with the state waves' final barrier
   }
@@ -1885,7 +1971,7 @@ namespace {
 // device holds its own copy; read through fr2_handoff_fault_count).
 __device__ int g_handoff_faults;
 std::atomic<int> g_spin_limit{1 << 20};
-std::atomic<bool> g_handoff_stall{false};
+std::atomic<int> g_handoff_stall{0};
 std::atomic<int> g_chunk_ring{1};
 std::atomic<int*> g_fault_ptr[64];
 }  // namespace
@@ -1903,10 +1989,10 @@ int* handoff_fault_word() {
   return ptr;
 }
 int handoff_spin_limit() { return g_spin_limit.load(std::memory_order_relaxed); }
-bool handoff_stall() { return g_handoff_stall.load(std::memory_order_relaxed); }
+int handoff_stall() { return g_handoff_stall.load(std::memory_order_relaxed); }
 bool chunk_ring_enabled() { return g_chunk_ring.load(std::memory_order_relaxed) != 0; }
 void set_chunk_ring(int on) { g_chunk_ring.store(on, std::memory_order_relaxed); }
-void set_handoff_stall(bool on) { g_handoff_stall.store(on, std::memory_order_relaxed); }
+void set_handoff_stall(int mode) { g_handoff_stall.store(mode, std::memory_order_relaxed); }
 void set_handoff_spin_limit(int polls) {
   g_spin_limit.store(polls < 0 ? (1 << 20) : polls, std::memory_order_relaxed);
 }
@@ -1919,8 +2005,23 @@ bool ring_contract(const SegArgs& p) {
          p.ro_out == nullptr;
 }
 
+// A unit's share: the state after piece 0, two blocks for each of pieces 1..P-2, the
+// saved start state, and P flags (rounded up to 16 bytes).
 int64_t split_workspace_floats(int nseg, int H, int pieces) {
-  return static_cast<int64_t>(nseg) * (3 * pieces - 2) * H * D * D;
+  const int64_t units = static_cast<int64_t>(nseg) * H;
+  return units * (2 * pieces - 2) * D * D + (units * pieces + 3) / 4 * 4;
+}
+// Points p's split at its workspace.
+static void set_split(SegArgs& p, int nseg, int pieces, int piece_len, int lead_len,
+                      float* workspace) {
+  const int64_t unit_floats = static_cast<int64_t>(nseg) * p.num_heads * D * D;
+  p.split_pieces = pieces;
+  p.split_len = piece_len;
+  p.split_lead = lead_len;
+  p.split_state = workspace;
+  p.split_saved = workspace + unit_floats;
+  p.split_summary = workspace + 2 * unit_floats;
+  p.split_flags = reinterpret_cast<int*>(workspace + (2 * pieces - 2) * unit_floats);
 }
 
 namespace {
@@ -1990,17 +2091,13 @@ int split_rule(int64_t units, int tokens, int& len) {
 int64_t train_split_workspace_floats(int nseg, int T, int H) {
   int len = 0;
   const int P = split_rule(static_cast<int64_t>(nseg) * H, T, len);
-  return P < 3 ? 0 : static_cast<int64_t>(nseg) * (2 * P - 3) * H * D * D;
+  return P < 3 ? 0 : split_workspace_floats(nseg, H, P);
 }
 void set_train_split(SegArgs& p, int nseg, int T, float* workspace) {
   int len = 0;
   const int P = split_rule(static_cast<int64_t>(nseg) * p.num_heads, T, len);
   if (P < 3 || workspace == nullptr) return;
-  p.split_pieces = P;
-  p.split_len = len;
-  p.split_lead = len;
-  p.split_state = workspace;
-  p.split_summary = workspace + static_cast<int64_t>(nseg) * p.num_heads * D * D;
+  set_split(p, nseg, P, len, len, workspace);
 }
 
 int launch_chunked(int dtype, const SegArgs& args, int nseg, int max_seqlen, hipStream_t s) {
@@ -2111,12 +2208,7 @@ int launch_chunked_split(int dtype, SegArgs p, int nseg, int pieces, int piece_l
   p.spin_limit = handoff_spin_limit();
   p.handoff_stall = handoff_stall();
   p.handoff_fault = handoff_fault_word();
-  p.split_pieces = pieces;
-  p.split_len = piece_len;
-  p.split_lead = lead_len;
-  // the states after piece 0, then the summaries of pieces 1..P-2
-  p.split_state = workspace;
-  p.split_summary = workspace + static_cast<int64_t>(nseg) * p.num_heads * D * D;
+  set_split(p, nseg, pieces, piece_len, lead_len, workspace);
   if (dtype == FR2_DTYPE_BFLOAT16)
     launch_split_kernels<IoBF16, kInfer>(p, nseg, s);
   else

@@ -62,12 +62,16 @@ struct SegArgs {
   // shorter; split_pieces is the most any segment has.  split_state holds the
   // state after each segment's first piece ([n, H, D, D]), split_summary the
   // final state from zero and the transition of its pieces 1..split_pieces-2
-  // ([n * (split_pieces - 2) + j - 1, 2, H, D, D]).
+  // ([n * (split_pieces - 2) + j - 1, 2, H, D, D]).  split_saved is the start
+  // state of a segment that is updated in place ([n, H, D, D]) and split_flags its
+  // blocks' failures ([n, H, split_pieces]; see split_flags_of in chunk.hip).
   int split_pieces = 0;
   int split_len = 0;
   int split_lead = 0;
   float* split_state = nullptr;
   float* split_summary = nullptr;
+  float* split_saved = nullptr;
+  int* split_flags = nullptr;
   // Row blocks (the training modes of the ring kernel on a chunk list): segment
   // n is the 16-token blocks [seq_blocks[n], seq_blocks[n + 1]), block j the
   // token rows row_blocks[2 j] .. + row_blocks[2 j + 1] (1 to 16 of them, each
@@ -84,8 +88,9 @@ struct SegArgs {
   int spin_limit = 1 << 20;
   int* handoff_fault = nullptr;
   // test hook: the key waves never publish their operators, so the state
-  // waves' waits give up (forces a real stall from the host)
-  bool handoff_stall = false;
+  // waves' waits give up (forces a real stall from the host): 1 in every block, 2
+  // in a split's later pieces but the last, 3 in its summaries
+  int handoff_stall = 0;
   // Fused kk / a-gate producer stage (chunked kernel only): `k` holds the
   // projected key, `a` the low-rank a-gate logits a12, `b` is unused; per
   // channel k_k, a0, k_a ([H, D]); the gated key is written to new_k.
@@ -190,8 +195,8 @@ void set_train_split(SegArgs& p, int nseg, int T, float* workspace);
 int* handoff_fault_word();
 int handoff_spin_limit();
 void set_handoff_spin_limit(int polls);   // negative: the default
-bool handoff_stall();
-void set_handoff_stall(bool on);
+int handoff_stall();
+void set_handoff_stall(int mode);
 bool chunk_ring_enabled();
 void set_chunk_ring(int on);
 int launch_chunked_split(int dtype, SegArgs p, int nseg, int pieces, int piece_len,

@@ -72,7 +72,10 @@ const char* fr2_last_error(void);
 /*
  * Count of chunked-kernel blocks that failed closed since the last reset on
  * the current device: a wave hand-off wait inside the block gave up, so the
- * block wrote NaN outputs and left its state untouched.  Waits for `stream`.
+ * block wrote NaN outputs and left its state untouched.  In a sequence split the
+ * state stays untouched when any block of its sequence and head failed, and the
+ * pieces whose start state depends on the failed block are NaN too (not counted
+ * again); the others hold their results.  Waits for `stream`.
  * No counterpart in the reference (its kernels have no bounded waits); the
  * fail-closed result mirrors the metadata path
  * (csrc/validation/recurrent_metadata.cu:24-132).
@@ -88,7 +91,8 @@ int fr2_debug_set_handoff_spin_limit(int32_t polls);
 /*
  * Test hook: while on (non-zero), the chunked kernel's key waves never
  * publish their operators, so each block's state waves stall at their first
- * operator wait and, after the spin limit, the block fails closed.  Forces a
+ * operator wait and, after the spin limit, the block fails closed.  2: only the
+ * later pieces of a sequence split but the last; 3: only its summaries.  Forces a
  * real stall from the host while every kernel still runs to its end.  No
  * counterpart in the reference.
  */
@@ -305,7 +309,7 @@ int fr2_wkv7_recurrent_fp32_forward_kk_gate_readout(
  * `stream`.  No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid allocation).  A plan whose workspace exceeds the
- * scratch (num_sequences * (3 pieces - 2) * num_heads * 16 KiB bytes) is
+ * scratch (num_sequences * num_heads * ((2 pieces - 2) * 16 KiB + 4 pieces) bytes) is
  * rejected with FR2_ERR_INVALID_ARGUMENT and an fr2_last_error() text.
  * Every call on one GPU shares that GPU's scratch: calls that overlap on one
  * GPU (two streams, two threads) race.
