@@ -213,7 +213,8 @@ int fr2_wkv7_prefill_split_plan(int32_t num_sequences, int32_t num_heads, int32_
 /*
  * A coarser plan for the same entries: pieces of at least 384 tokens in
  * multiples of 32, at most 256/units + 1 of them, piece 0 about 1.05x the
- * others.  fr2_wkv7_prefill_split_plan is the faster choice.
+ * others.  Reports num_sequences * (3 pieces - 2) * num_heads * 16 KiB, more than the
+ * entries need.  fr2_wkv7_prefill_split_plan is the faster choice.
  */
 int fr2_wkv7_recurrent_fp32_split_plan(int32_t num_sequences, int32_t num_heads,
                                        int32_t head_size, int32_t max_seqlen,
