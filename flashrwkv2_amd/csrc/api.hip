@@ -960,6 +960,15 @@ extern "C" int fr2_wkv7_statetune_padded_backward(
 
 namespace {
 constexpr int32_t kMaxRowSequences = 65535;
+// Lists whose blocks, every sequence filled up to the one with the most, hold more
+// than this many times their tokens (many tiny chunks, one long sequence among many
+// short ones) stay on the token-serial kernels.  Those compute in fp32 throughout,
+// the chunked ones split their operands in two bf16 terms: against fp64, one
+// sequence of 1 024 tokens among 14 of 33, final state and boundaries 1.1e-7 /
+// 2.7e-6 (token-serial / row blocks), sa 1.4e-7 / 5.7e-6, dL/dS0 1.0e-7 / 2.7e-6.
+// Below the line the chunked kernels have always run, and y and the token gradients
+// are rounded to bf16 either way.
+constexpr int64_t kMaxRowFill = 4;
 }  // namespace
 
 // Lays a StateTune chunk list (host arrays) out as row blocks for
@@ -970,9 +979,9 @@ constexpr int32_t kMaxRowSequences = 65535;
 //   chunk_seq [C], chunk_block [C], seq_first_chunk [B]
 // and info = {blocks, spans, blocks per span, most blocks of a sequence}.
 // Returns the table's length; 0 when the list does not suit it (offsets that do
-// not cover the list, rows out of range or in two chunks, no tokens, more than
-// four times the tokens in blocks: many tiny chunks run faster token-serial, or more
-// sequences, chunks or spans than a grid holds); -1 for an invalid argument, -2 when `capacity` (ints) is too small.
+// not cover the list, rows out of range or in two chunks, no tokens, more
+// sequences, chunks or spans than a grid holds, or kMaxRowFill); -1 for an invalid
+// argument, -2 when `capacity` (ints) is too small.
 // 4 * (T / 16 + C) + 3 * (B + 1) + 2 * C ints always suffice.
 extern "C" int64_t fr2_wkv7_statetune_rows_plan(
     const int32_t* sequence_chunk_offsets, const int32_t* chunk_token_starts,
@@ -989,13 +998,17 @@ extern "C" int64_t fr2_wkv7_statetune_rows_plan(
   if (off[0] != 0 || off[B] != C) return 0;
   for (int b = 0; b < B; ++b)
     if (off[b + 1] < off[b] || off[b + 1] > C) return 0;
-  int64_t used = 0, blocks = 0;
-  for (int c = 0; c < C; ++c) {
-    if (st[c] < 0 || en[c] < st[c] || en[c] > total_tokens) return 0;
-    used += en[c] - st[c];
-    blocks += (static_cast<int64_t>(en[c]) - st[c] + 15) / 16;
+  int64_t used = 0, blocks = 0, longest = 0;
+  for (int b = 0; b < B; ++b) {
+    const int64_t before = blocks;
+    for (int c = off[b]; c < off[b + 1]; ++c) {
+      if (st[c] < 0 || en[c] < st[c] || en[c] > total_tokens) return 0;
+      used += en[c] - st[c];
+      blocks += (static_cast<int64_t>(en[c]) - st[c] + 15) / 16;
+    }
+    longest = std::max(longest, blocks - before);
   }
-  if (used == 0 || used > total_tokens || 16 * blocks > 4 * used) return 0;
+  if (used == 0 || used > total_tokens || 16 * B * longest > kMaxRowFill * used) return 0;
   try {
     // rows in two chunks: neighbours in the order of their first rows (mostly
     // the list's own order)

@@ -43,7 +43,8 @@ def test_rows_match_the_padded_grid(seed):
     offsets, starts, ends, T = _random_list(rng)
     H = int(rng.choice([1, 4, 64]))
     grid, rows, B, n = _both(offsets, starts, ends, max(T, 1), H)
-    if grid is None:   # (the grid also pads every sequence to the longest)
+    assert (grid is None) == (rows is None)
+    if grid is None:
         return
     Tp, row_source, chunk_seq, pstart, first = grid
     table, (blocks, spans, every, most) = rows
@@ -84,6 +85,10 @@ def test_more_sequences_or_chunks_than_a_grid_holds(B, H):
     ([1, 1, 2], [0, 64], [64, 128], 128),
     ([0, 9], list(range(9)), list(range(1, 10)), 9),   # nine one-token chunks: 16x blocks
     ([0, 1], [0], [0], 16),                        # no tokens
+    # one long sequence among short ones: filled up to it, more than four times the
+    # tokens, which the fp32 token-serial kernels keep
+    ([0, 2, 3, 4, 5, 6, 7], [0, 128, 256, 257, 258, 259, 260],
+     [128, 256, 257, 258, 259, 260, 261], 261),
 ])
 def test_lists_that_are_refused(offsets, starts, ends, T):
     grid, rows, _, _ = _both(offsets, starts, ends, T)
