@@ -215,9 +215,9 @@ def test_dispatch_query_reports_the_policy(lib, n, h, d, total, maxlen, want):
 ])
 def test_wide_head_rule_follows_the_measured_costs(lib, n, h, d, total, maxlen, chunked):
     import ctypes
+    import importlib
 
-    from flashrwkv2_amd import _C
-
+    _C = importlib.import_module("flashrwkv2_amd._C")   # (the package sets it only with a GPU)
     assert _C.dispatch_kernel_name(n, h, d, total, maxlen).startswith("chunk_wide") == chunked
     got = ctypes.c_int32(-1)
     assert lib.fr2_wkv7_recurrent_fp32_wide_chunked(n, h, d, total, maxlen,
