@@ -166,14 +166,15 @@ def test_config1_shape_fp16():
 
 
 def test_few_long_fp16_sequences_take_the_split():
-    """Few long fp16 sequences: the library's plan splits them by sequence, so
-    the gate runs as its own kernel and the recurrence takes the split."""
+    """Few long fp16 sequences, where the split outruns one block per unit: the
+    gate runs as its own kernel and the recurrence takes the split."""
     require_gpu()
     from flashrwkv2_amd import _C
 
     print("case kk-gate long fp16 split", flush=True)
     c = _case([3000], 8, torch.float16, seed=21)
-    assert _C.split_plan(1, 8, 64, 3000)[0] > 1
+    assert _C._gate_runs_apart(1, 8, 64, 3000, readout=False)
+    assert _C.prefill_plan(1, 8, 64, 3000)[0] > 1
     y, pool, new_k = _run(c, 1.0)
     ey, epool, ek = _expected(c, 1.0)
     assert_output_close(y, ey)

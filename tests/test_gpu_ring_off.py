@@ -1,11 +1,10 @@
 """The ring variant of the workgroup chunked kernel is the default for every
 inference contract (the bf16-state pool, rl_infctx chunk lists, the fused
-kk / a-gate stage, the real and summary passes of the sequence split).  With
-the ring switched off (`_C._set_chunk_ring(False)`) the same entries run on
-the key-half kernel instead; these cases re-run representative parity tests
-of each entry in that configuration, so both kernels stay checked against
-the fp64 oracle.  The training backward's value pass (the reverse mode) is
-on the ring as well, and is re-run here on the key-half kernel too."""
+kk / a-gate stage) and for the training passes.  With the ring switched off
+(`_C._set_chunk_ring(False)`) the same entries run on the key-half kernel
+instead; these cases re-run representative parity tests of each entry in that
+configuration, so both kernels stay checked against the fp64 oracle.  The
+sequence split has the ring's form only and does not look at the switch."""
 
 from __future__ import annotations
 
@@ -17,7 +16,7 @@ import test_gpu_other_entries as entry_tests
 import test_gpu_pretrain_backward as bwd_tests
 import test_gpu_split as split_tests
 import test_gpu_statetune as st_tests
-from wkv7_testlib import require_gpu
+from wkv7_testlib import make_case, require_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -47,10 +46,28 @@ def test_fused_kk_gate_on_the_key_half_kernel(ring_off, dtype):
     kk_tests.test_fused_kk_gate_matches_the_two_stage_oracle(dtype, (300, 64, 96, 41), 4, True)
 
 
-@pytest.mark.parametrize("lengths,pieces", [((700, 64, 1, 129, 1024), 4),
-                                            ((700, 64, 1, 129, 1024), (4, 320))])
-def test_split_summary_on_the_key_half_kernel(ring_off, lengths, pieces):
-    split_tests.test_split_matches_oracle_and_unsplit(lengths, pieces, torch.bfloat16)
+@pytest.mark.parametrize("pieces", [4, (4, 320)])
+def test_split_does_not_look_at_the_switch(ring_off, pieces):
+    """The same pieces with the ring off and on: the same bits, while the unsplit
+    kernel's, which does look at it, differ (they sum in another order)."""
+    C = require_gpu()
+    case = make_case(dtype=torch.bfloat16, head_size=64, lengths=(700, 64, 1, 129, 1024),
+                     num_heads=2, seed=5)
+    runs = {}
+    for on in (False, True):
+        C._set_chunk_ring(on)
+        for kernel in (split_tests.SPLIT, split_tests.CHUNKED):
+            pool = case["state_pool"].clone()
+            y = split_tests._forced(C, kernel, case, pool,
+                                    pieces=pieces if kernel == split_tests.SPLIT else None)
+            runs[kernel, on] = y, pool
+    for a, b in zip(runs[split_tests.SPLIT, False], runs[split_tests.SPLIT, True]):
+        assert torch.equal(a, b)
+    assert not torch.equal(runs[split_tests.CHUNKED, False][1], runs[split_tests.CHUNKED, True][1])
+
+
+def test_pretrain_forward_on_the_key_half_kernel(ring_off):
+    entry_tests.test_pretrain_forward_matches_oracle(2, 96, 2, 64, True)   # (too short to split)
 
 
 def test_pretrain_backward_value_pass_on_the_key_half_kernel(ring_off):

@@ -1,12 +1,12 @@
 """GPU parity of the sequence-split chunked prefill (few long sequences).
 
-A split run cuts every sequence into pieces: a summary pass computes each
-piece's zero-start final state F and transition Phi, a combine kernel chains
-S(j+1) = Phi_j S(j) + F_j, and the chunked kernel runs the pieces from those
-start states.  The classic split (equal pieces) chains from the slot state;
-the pipelined split runs piece 0 (its own length) from the slot state on a
-second stream next to the summary pass and chains from its end state.  The results must match the fp64 oracle on exactly the
-kernel's inputs with the same gates as the unsplit kernels (relative RMSE
+A split run cuts every sequence into pieces, in two launches: piece 0 runs
+from the slot state next to the summaries of the later pieces but the last
+(zero-start final state F and transition Phi), then pieces 1 and up run, each
+from its start state S(j+1) = Phi_j S(j) + F_j carried on from piece 0's end.
+Plans are given as a number of equal pieces or as (pieces, piece 0's length).
+The results must match the fp64 oracle on exactly the kernel's inputs with the
+same gates as the unsplit kernels (relative RMSE
 2e-3 from tests/fixtures/tolerances-v1.json:9-12 of the reference, plus
 |dy| <= 2e-2 max(1, |y|) and ||dS|| / ||S|| <= 1e-3 per (slot, head)), and
 agree with the unsplit chunked kernel to fp32-level accuracy.
@@ -63,8 +63,8 @@ def _close_to_unsplit(y_split, y_chunk, p_split, p_chunk, active):
     ((700, 64, 1, 129, 1024), 4),       # sequences of 1..4 pieces, ragged last pieces
     ((2000, 33), 3),
     ((96, 96, 96), 3),                  # pieces of 32 tokens
-    # pipelined split: (pieces, piece 0's length)
-    ((1024,), (2, 512)),                # no summary pass, no combine
+    # (pieces, piece 0's length)
+    ((1024,), (2, 512)),                # no summaries
     ((1024,), (4, 352)),
     ((700, 64, 1, 129, 1024), (4, 320)),   # sequences ending inside piece 0 and later
     ((2000, 33), (3, 1024)),
@@ -95,11 +95,17 @@ def test_split_matches_oracle_and_unsplit(lengths, pieces, dtype):
 
 
 def test_public_call_splits_a_long_single_sequence():
-    """B = 1 prefill (4 heads): the public entry takes the split by itself
-    (the plan cuts it into pieces of at least 384 tokens) and matches the oracle."""
+    """B = 1 prefill (4 heads): the public entry takes the split by itself, at
+    the plan it asks for (the coarser plan of the C interface is checked next to
+    it), and matches the oracle."""
     C = require_gpu()
     from flashrwkv2_amd import _C as CC
 
+    pieces, plen, lead, _ = CC.prefill_plan(1, 4, 64, 8192)
+    assert pieces >= 3 and lead == plen and plen % 16 == 0
+    assert (pieces - 1) * plen < 8192 <= pieces * plen
+    assert CC.prefill_plan(8, 32, 64, 4096)[0] == 1    # 256 units, no split
+    assert CC.dispatch_kernel_name(1, 4, 64, 8192, 8192).startswith("split:")
     pieces, plen, lead, _ = CC.split_plan(1, 4, 64, 8192)
     assert pieces >= 3 and plen >= 384 and lead >= plen and lead % 32 == 0 == plen % 32
     assert lead + (pieces - 2) * plen < 8192 <= lead + (pieces - 1) * plen
@@ -117,8 +123,8 @@ def test_public_call_splits_a_long_single_sequence():
 
 
 def test_split_fails_closed_on_invalid_metadata():
-    """Device-detected metadata errors: NaN output, state pool untouched, on
-    every kernel of the split (summary, combine, pieces)."""
+    """Device-detected metadata errors: NaN output, state pool untouched, in
+    both launches of the split."""
     C = require_gpu()
     case = make_case(dtype=torch.bfloat16, lengths=(2048,))
     pool = case["state_pool"]
@@ -157,7 +163,7 @@ def test_split_under_graph_capture_with_live_metadata():
     n_seq = torch.full((1,), 2, device=dev, dtype=torch.int32)
     live = dict(state_pool_size=slots_n, token_capacity=4000, sequence_capacity=2,
                 max_seqlen_capacity=4000, num_active_tokens=n_tok, num_active_sequences=n_seq)
-    assert CC.split_plan(2, 2, 64, 4000)[0] >= 3           # the capacity plan splits
+    assert CC.prefill_plan(2, 2, 64, 4000)[0] >= 3         # the capacity plan splits
     y_ref, pool_ref = oracle_expect(case)
     active = case["state_indices"].long()
     stream = torch.cuda.Stream()

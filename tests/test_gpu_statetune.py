@@ -286,7 +286,7 @@ def test_statetune_uniform_layout_runs_chunked_kernels(B, per_seq, length, scale
 
 def test_statetune_uniform_autograd_and_fallbacks():
     """The public function takes the chunked path on the uniform layout and
-    the padded chunked path on a ragged layout of the same tokens; both match
+    the row blocks on a ragged layout of the same tokens; both match
     the oracle and each other."""
     require_gpu()
     g = torch.Generator().manual_seed(77)
@@ -326,9 +326,9 @@ def _ragged_meta(B, per_seq, rng, gap=0):
 
 
 @pytest.mark.parametrize("B,per_seq,H,gap", [(3, 700, 2, 0), (2, 1500, 3, 37)])
-def test_statetune_ragged_chunk_list_runs_the_padded_chunked_path(B, per_seq, H, gap):
+def test_statetune_ragged_chunk_list_runs_as_row_blocks(B, per_seq, H, gap):
     """A ragged chunk list at D = 64 in bf16 runs on the chunked MFMA kernels
-    over the padded grid (the forward returns the grid's tables); forward,
+    as row blocks (the forward returns their table and sizes); forward,
     final state, boundaries and every gradient match the fp64 oracle and the
     token-serial kernels on the same inputs."""
     C = require_gpu()
@@ -344,15 +344,18 @@ def test_statetune_ragged_chunk_list_runs_the_padded_chunked_path(B, per_seq, H,
           flush=True)
     dy = torch.randn((T, H, D), generator=g).to(torch.bfloat16).cuda()
     dfin = torch.randn((B, H, D, D), generator=g).cuda()
-    # the forward takes the padded path (tables returned for the backward)
+    # the forward takes the row blocks (what it returns for the backward)
     st = state0.clone()
     probe = C.statetune_tmix_wkv7_recurrent_fp32io16_forward(
         *meta, st, *vals, torch.empty_like(vals[3]),
         torch.empty((meta[1].numel(), H, D, D), device="cuda"),
         torch.empty((T, H, D), device="cuda"), 1.0)
-    assert isinstance(probe, tuple) and len(probe) == 3
+    snapshots, table, sizes = probe
+    blocks = sum(-(-int(n) // 16) for n in (meta[2] - meta[1]).tolist())
+    assert tuple(snapshots.shape) == (blocks, H, D, D) and sizes[0] == blocks
+    assert table.is_cuda and table.dtype == torch.int32
     runs = {}
-    for name, serial in (("padded", False), ("serial", True)):
+    for name, serial in (("rows", False), ("serial", True)):
         CC._statetune_force_serial = serial
         try:
             state, leaves, (y, fin, bnd, sa) = _run(state0, meta, vals, 1.0)
@@ -364,7 +367,7 @@ def test_statetune_ragged_chunk_list_runs_the_padded_chunked_path(B, per_seq, H,
     ref = _oracle(state0, meta, vals, 1.0, dy=dy, dfinal=dfin)
     starts, ends = meta[1].cpu().numpy(), meta[2].cpu().numpy()
     used = np.concatenate([np.arange(s0, e0) for s0, e0 in zip(starts, ends)])
-    got = runs["padded"]
+    got = runs["rows"]
     _check_strong({k: got[k][used] for k in ("y", "sa")}, {k: ref[k][used] for k in ("y", "sa")},
                   ("y", "sa"), rel=5e-3)
     for key in ("state", "boundary"):

@@ -23,7 +23,7 @@ SHAPES = [
     (1, 4096, 2, True),
     (2, 1088, 64, True),     # 128 units: three pieces
     (1, 256, 2, False),      # too short to gain: the ring kernel, whole
-    (1, 32, 200, False),     # above the ring forward's unit limit
+    (1, 1088, 129, False),   # one unit too many for two pieces after the first
 ]
 
 
