@@ -525,7 +525,7 @@ def time_kk_fused(torch, flashrwkv2_amd, steps: int, serving: bool = False):
         w = workloads.config(1, "cuda", dtype=torch.float16)
         rec_kernel, kk_kernel, ro_kernel = (
             "chunk64r_kernel<IoF16>", "chunk64r_kernel<IoF16,kk>",
-            "chunk64_kernel<IoF16,false,false,false,true,true>")
+            "chunk64_kernel<IoF16,false,false,true,true>")
         name = "cfg1_prefill_B8_T4096_H32_fp16_kk_gate"
     T, H, D = w.total_tokens, w.num_heads, 64
     C = H * D
@@ -649,7 +649,7 @@ def time_long_context(torch, flashrwkv2_amd, steps: int):
                    "chunk64r_kernel pieces 1..P-1",
         "pieces": pieces, "piece_len": piece_len, "lead_len": lead_len, "workspace_bytes": ws,
         "roofline": roofline_obj(nbytes, ms, measured_traffic(
-            "split:lead+summary+combine+pieces", w.name)),
+            "split:lead+summary,pieces", w.name)),
         "unsplit": {"ms_per_step": round(unsplit_ms, 4),
                     "tokens_per_s": round(w.total_tokens / (unsplit_ms * 1e-3), 1),
                     "kernel": "chunk64r_kernel<IoBF16> (one block per head)",
@@ -843,7 +843,7 @@ def time_other_paths(torch, flashrwkv2_amd, w, steps: int):
                      "flops_per_token_head": FLOPS_PER_TOKEN_HEAD},
         },
         "rl_infctx_forward": {
-            "kernel": "chunk64_kernel<IoBF16,false> over each sequence's chunk list",
+            "kernel": "chunk64r_kernel<IoBF16> over each sequence's chunk list",
             "chunk_size": 16, "kernel_ms": round(f_ms, 4),
             "tokens_per_s": round(T / (f_ms * 1e-3), 1),
             "roofline": roofline_obj(io + 2 * B * H * STATE_BYTES, f_ms),
@@ -893,7 +893,7 @@ def time_chunk_bf16_state(torch, flashrwkv2_amd, w, steps: int):
               + 2 * w.state_indices.numel() * w.num_heads * STATE_BYTES // 2)   # bf16 state
     return {"workload": w.name + "_bf16_state", "ms_per_step": round(ms, 5),
             "tokens_per_s": round(w.total_tokens / (ms * 1e-3), 1),
-            "kernel": "chunk64_kernel<IoBF16,false> (bf16 state load/store)",
+            "kernel": "chunk64r_kernel<IoBF16> (bf16 state load/store)",
             "roofline": roofline_obj(nbytes, ms)}
 
 
@@ -901,7 +901,7 @@ def _bwd_traffic(B, T, H):
     """Measured HBM bytes of the two backward kernels (PMC, committed), when
     the workload is the measured one."""
     wl = f"cfg1_shape_training_B{B}_T{T}_H{H}"
-    parts = [measured_traffic(k, wl) for k in ("chunk64r_kernel<IoBF16,false,true>", "key_chunk_kernel")]
+    parts = [measured_traffic(k, wl) for k in ("chunk64r_kernel<IoBF16,false,kBwd>", "key_chunk_kernel")]
     return None if any(x is None for x in parts) else sum(parts)
 
 
@@ -977,8 +977,8 @@ def time_pretrain_training(torch, w, steps: int):
         "backward_algorithmic_bytes": bwd_bytes,
         "backward_roofline": roofline_obj(bwd_bytes, bwd_ms, _bwd_traffic(B, T, H)),
         "gradients_finite": ok,
-        "kernels": ["chunk64_kernel<IoBF16,true> (forward: y, sa, boundary)",
-                    "chunk64r_kernel<IoBF16,false,true> (value pass: dv, dsa, P snapshots)",
+        "kernels": ["chunk64r_kernel<IoBF16,false,kFwd> (forward: y, sa, boundary)",
+                    "chunk64r_kernel<IoBF16,false,kBwd> (value pass: dv, dsa, P snapshots)",
                     "key_chunk_kernel (key pass: dr, dw, dk, db, da)"],
     }
 
@@ -999,9 +999,9 @@ def time_statetune_ragged(torch, w, steps: int):
     """StateTune on the config-1 shape (8 x 4096 tokens, H = 32) over a
     ragged chunk list: chunks of seeded random lengths 1..700 (most not a
     multiple of 16), a few empty, and 40 tokens of each sequence in no chunk.
-    Through the public `_C` entries (the forward builds the padded grid on
+    Through the public `_C` entries (the forward builds the row-block table on
     the host from the chunk metadata, then runs the chunked MFMA kernels;
-    the backward reuses the grid), per call, HIP events and wall clock; the
+    the backward reuses the table), per call, HIP events and wall clock; the
     token-serial kernels on the same list for comparison."""
     import numpy as np
 
@@ -1057,9 +1057,9 @@ def time_statetune_ragged(torch, w, steps: int):
         finally:
             CC._statetune_force_serial = False
         out[name] = {"forward_ms": round(f_ms, 4), "backward_ms": round(b_ms, 4),
-                     # the chunked forward returns its padded-grid plan for the
+                     # the chunked forward returns its row-block table for the
                      # backward; the token-serial one returns nothing
-                     "path": "padded_chunked" if res["snap"] is not None else "token_serial"}
+                     "path": "row_blocks" if res["snap"] is not None else "token_serial"}
     out["gradients_finite"] = all(bool(torch.isfinite(t).all()) for t in (*grads, g0))
     del state, dy, y, boundary, sa, grads, res
     torch.cuda.empty_cache()
@@ -1164,8 +1164,8 @@ def time_statetune_training(torch, w, steps: int, chunk_len: int = 1024):
                          "forward_roofline": roofline_obj(fwd_bytes, sf),
                          "backward_roofline": roofline_obj(bwd_bytes, sb)},
         "gradients_finite": ok,
-        "kernels": ["chunk64_kernel<IoBF16,true> (forward) + st_gather_kernel (boundaries)",
-                    "chunk64r_kernel<IoBF16,false,true> + first_token_kernel + key_chunk_kernel "
+        "kernels": ["chunk64r_kernel<IoBF16,false,kFwd> (forward) + st_gather_kernel (boundaries)",
+                    "chunk64r_kernel<IoBF16,false,kBwd> + first_token_kernel + key_chunk_kernel "
                     "(backward)",
                     "token-serial: st_forward_kernel, st_value_kernel, st_key_kernel"],
     }

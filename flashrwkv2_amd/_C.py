@@ -122,9 +122,9 @@ def _set_handoff_stall(on: int) -> None:
 
 def _set_chunk_ring(on: bool) -> None:
     """Test hook: selects the workgroup chunked kernel's variant for later
-    fp32-state launches: True = one key wave per whole chunk over a ring of
-    four chunk operator blocks (the default), False = two key waves per chunk
-    with the token-token blocks summed through LDS."""
+    launches that are not split: True = one key wave per whole chunk over a
+    ring of chunk operator blocks (the default), False = two key waves per
+    chunk with the token-token blocks summed through LDS."""
     N.check(N.load().fr2_debug_set_chunk_ring(int(bool(on))), "fr2_debug_set_chunk_ring")
 
 

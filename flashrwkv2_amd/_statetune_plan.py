@@ -1,6 +1,7 @@
 """Host-side layouts of StateTune's ragged chunk lists for the chunked kernels:
 row blocks (fr2_wkv7_statetune_rows_forward / _backward, what the package runs)
-and the padded grid (fr2_wkv7_statetune_padded_forward / _backward)."""
+and the padded grid (fr2_wkv7_statetune_padded_forward / _backward, for callers of
+the C interface; the package uses it only to test the row blocks against)."""
 
 from __future__ import annotations
 

@@ -332,8 +332,8 @@ extern "C" int fr2_wkv7_recurrent_fp32_forward_split(
 // The array's name is a host-side stand-in for the device symbol: host code
 // uses only the device address hipGetSymbolAddress returns, looked up once
 // per device with that device current and kept in g_scratch_ptr.
-// No clearing is needed: every float of the workspace a call reads was
-// written earlier in the same call (summaries, then chained start states).
+// No clearing is needed: the call's second launch reads only what its first one
+// wrote (piece 0's end states, summaries, failure words).
 // Calls that overlap on one GPU share the array and race.
 // ---------------------------------------------------------------------------
 constexpr int64_t kNoAllocScratchFloats = int64_t{4} << 20;   // 16 MiB
@@ -376,7 +376,8 @@ extern "C" int fr2_wkv7_recurrent_fp32_forward_split_noalloc(
   if (need > kNoAllocScratchFloats) {
     fr2::set_last_error(
         "fr2_wkv7_recurrent_fp32_forward_split_noalloc: the split's workspace exceeds the "
-        "16 MiB no-allocation scratch (num_sequences * num_heads * ((2 pieces - 2) * 16 KiB + 4 pieces))");
+        "16 MiB no-allocation scratch (num_sequences * num_heads * "
+        "((2 pieces - 2) * 16 KiB + 4 pieces))");
     return FR2_ERR_INVALID_ARGUMENT;
   }
   float* ws = scratch_address();
@@ -384,7 +385,6 @@ extern "C" int fr2_wkv7_recurrent_fp32_forward_split_noalloc(
     fr2::set_last_error("fr2_wkv7_recurrent_fp32_forward_split_noalloc: scratch lookup failed");
     return FR2_ERR_LAUNCH;
   }
-  // one stream: the pipelined split's second stream would need events
   return fr2_wkv7_recurrent_fp32_forward_split(
       query_start_loc, state_indices, status, num_sequences, num_heads, head_size, total_tokens,
       max_seqlen, dtype, state, r, decay_logits, decay_bias, k, v, a, b, output, scale, pieces,

@@ -1997,9 +1997,9 @@ void set_handoff_spin_limit(int polls) {
   g_spin_limit.store(polls < 0 ? (1 << 20) : polls, std::memory_order_relaxed);
 }
 
-// the ring variant covers the inference contracts (fp32 or bf16 state,
-// packed, uniform or chunk-list segments); the training outputs (boundary
-// snapshots, sa) and the fused read-out stay on chunk64_kernel
+// whether an inference call (fp32 or bf16 state, packed, uniform or chunk-list
+// segments) runs on the ring variant: all but the fused read-out do, which stays on
+// chunk64_kernel, as does everything unsplit with the ring switched off
 bool ring_contract(const SegArgs& p) {
   return chunk_ring_enabled() && p.boundary == nullptr && p.sa_out == nullptr &&
          p.ro_out == nullptr;

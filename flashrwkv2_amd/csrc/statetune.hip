@@ -527,6 +527,8 @@ __global__ __launch_bounds__(256) void st_gather_kernel(int H, int nck, int chun
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 // ---- ragged chunk lists on the chunked kernels (the padded layout) ----
+// For callers of the C interface, and the form the row blocks are tested against;
+// the package's own calls run the row blocks.
 // Each sequence's chunks are laid out back to back in a [B, Tp] token grid,
 // every chunk starting on a 16-token boundary; the rows in between (and at
 // the end of a sequence) hold identity tokens (r = k = v = a = b = 0 and a

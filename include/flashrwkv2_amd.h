@@ -627,7 +627,9 @@ int fr2_wkv7_statetune_uniform_backward(
 
 /*
  * StateTune over any chunk list (ragged, empty or gapped chunks) at
- * head_size 64 with bf16 tokens, on the chunked MFMA kernels: each
+ * head_size 64 with bf16 tokens, on the chunked MFMA kernels, over a copy of the
+ * tokens (fr2_wkv7_statetune_rows_forward below needs none and is the faster
+ * choice; the package's own calls take it): each
  * sequence's chunks are laid out back to back in a [batch, padded_tokens]
  * token grid (padded_tokens a multiple of 16), every chunk starting on a
  * 16-token boundary, with identity tokens in between (zero r, k, v, a, b and
