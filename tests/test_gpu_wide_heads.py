@@ -86,6 +86,33 @@ def test_wide_training_forward_outputs(batch, tokens_, heads, head_size):
     assert relative_rmse(to_np(bnd), bnd_ref) <= STATE_REL
 
 
+@pytest.mark.parametrize("head_size", [128, 256])
+def test_wide_rl_infctx_replay(head_size):
+    """Chunks from their own start states, with decay bias and scale: y and sa, and
+    the start states untouched."""
+    C = require_gpu()
+    lengths, heads = (33, 17, 64, 1), 2
+    assert C.dispatch_kernel_name(len(lengths), heads, head_size, sum(lengths),
+                                  0).startswith("chunk_wide_kernel")
+    case = make_case(dtype=torch.bfloat16, head_size=head_size, lengths=lengths, num_heads=heads,
+                     with_decay_bias=True, seed=head_size + 1)
+    g = torch.Generator().manual_seed(head_size)
+    starts = torch.randn((len(lengths), heads, head_size, head_size), generator=g).cuda()
+    before, cu = starts.clone(), case["cu_seqlens"]
+    out, sa = torch.empty_like(case["v"]), torch.empty(case["v"].shape, device="cuda")
+    C.rl_infctx_tmix_wkv7_chunk_fp32io16_backward_replay(
+        cu[:-1].contiguous(), cu[1:].contiguous(), starts, *tokens(case), out, sa, 0.75,
+        case["decay_bias"])
+    torch.cuda.synchronize()
+    y_ref, _, sa_ref, _ = oracle.wkv7_f64(
+        *(to_np(t) for t in tokens(case)), cu_seqlens=to_np(cu),
+        state_indices=np.arange(len(lengths), dtype=np.int32), state_pool=to_np(starts),
+        decay_bias=to_np(case["decay_bias"]), scale=0.75, want_sa=True)
+    assert_output_close(out, y_ref)
+    assert relative_rmse(to_np(sa), sa_ref) <= STATE_REL
+    assert torch.equal(starts, before)
+
+
 def _token_serial_f32(x):
     """Final states and sa of [B, T, H, D] inputs from a zero state, token by token
     in fp32 (sums over keys in pairs)."""
